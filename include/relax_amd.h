@@ -86,13 +86,17 @@ enum { RELAX_AMD_KERNEL_AUTO = 0, RELAX_AMD_KERNEL_TWO_WALK = 1, RELAX_AMD_KERNE
  * Process-wide, read atomically at each launch; returns the previous choice, or RELAX_AMD_EINVAL.  No counterpart
  * in the reference: it exists for tests and measurements.
  *
- * The one-shot kernels of the actor step and of the reverse-KL step each keep their exchange ring (1.5 MB, plus 8 MB
- * for the logits gathered at a row's top-K ids / 2.5 MB) in static arrays of the library, one copy per GPU and process.  Launches of the same entry point that overlap on
- * one GPU (two streams of one process) must not both take that kernel: they could overwrite each other's slots, which
- * the kernel notices (bounded waits) and reports as NaN log-probs (NaN KL) rather than wrong numbers.  Launches in stream order, captured graphs and their replays
- * are fine (the tags that tell one launch's partial sums from another's come from a counter in device memory that a
- * small kernel in front of each launch advances); the first call on a GPU looks the ring's address up
- * (hipGetSymbolAddress), so make one call outside a capture first.
+ * The one-shot kernels of the actor step and of the reverse-KL step exchange through rings in static arrays of the
+ * library, one copy per GPU and process: six rings each (1.5 MB, plus 8 MB for the logits gathered at a row's top-K ids /
+ * 2.5 MB; 58 + 15 MB).  Calls may come from any threads and streams and may overlap.  Each of the first four streams of a
+ * GPU that make such calls has a ring; the calls of all other streams (and of a per-thread default stream) share one, on
+ * which a step waits for the step before it (an event).  A stream that is destroyed should be idle by then: another
+ * stream may get its handle and with it its ring.  Every launch has tags of its own for the words it exchanges, so
+ * launches that do meet on a ring end in bounded waits and NaN log-probs (NaN KL), not in each other's numbers.
+ * Captured launches (up to 4096 per process, GPU and entry point, two-walk or resident kernels beyond) share a ring and
+ * take their tags on the device, new ones at each replay; replays of captured steps of one entry point that overlap on a
+ * GPU are such a meeting: keep them in one order, or capture with TWO_WALK.  The first call on a GPU looks the arrays'
+ * addresses up (hipGetSymbolAddress), so make one call outside a capture first.
  */
 int relax_amd_set_kernel_choice(int choice);
 /*

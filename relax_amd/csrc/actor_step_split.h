@@ -19,6 +19,9 @@ constexpr int kSplit = 1024 / kSplitThreads;
 constexpr size_t kRingWords = size_t(kRing) * kSlotWords;
 constexpr size_t kTopkRingWords = size_t(kRing) * RELAX_AMD_FUSED_TOPK_MAX;
 
+// the ring and the tags of an actor step about to be enqueued (actor_step_split.hip)
+int open_split_exchange(ExchangeLaunch& x, hipStream_t stream, int64_t n_rows, bool own_ring_only);
+
 // scan_absorb() over the values of kScanUnroll raw vectors (as in actor_step_resident.hip: same arithmetic, same
 // order)
 // KEEP: whether the second walk may use the values the first one unpacked (32 registers for 16-bit rows); without, the
@@ -74,12 +77,13 @@ __device__ __forceinline__ void split_publish(unsigned long long* slot, unsigned
 // workgroup of that many waves does in scan_block_merge().
 template <int ROW_WAVES = kRowWaves>
 __device__ __forceinline__ SoftmaxAcc split_collect(const unsigned long long* slot, unsigned tag, int tid,
-                                                    unsigned max_polls, unsigned* status, bool& any_gave_up) {
+                                                    unsigned max_polls, unsigned* status, unsigned first_tag,
+                                                    bool& any_gave_up) {
   float word = 0.f;
   bool gave_up = false;
-  if (tid < ROW_WAVES * 3) gave_up = !exchange_wait(slot + tid, tag, max_polls, status, word);
+  if (tid < ROW_WAVES * 3) gave_up = !exchange_wait(slot + tid, tag, max_polls, status, first_tag, word);
   any_gave_up = __any(gave_up);
-  if (any_gave_up && tid == 0) exchange_report_give_up(status);
+  if (any_gave_up && tid == 0) exchange_report_give_up(status, first_tag);
   auto of_lane = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(word), l)); };
   SoftmaxAcc whole{of_lane(0), of_lane(1), of_lane(2)};
 #pragma unroll
@@ -120,7 +124,8 @@ void actor_step_split_kernel(
     const int64_t* __restrict__ targets, float c, float inv_t, relax_amd_policy_loss_args a, float grad_scale,
     float* __restrict__ log_prob, float* __restrict__ entropy, float* __restrict__ lse_out,
     float* __restrict__ spx_out, T* __restrict__ dlogits, int64_t d_stride, unsigned long long* __restrict__ ring,
-    unsigned long long* __restrict__ topk_ring, unsigned laps, unsigned max_polls, unsigned wait_tag_offset) {
+    unsigned long long* __restrict__ topk_ring, unsigned tag_base, const unsigned* __restrict__ tag_word,
+    unsigned max_polls, unsigned wait_tag_offset) {
   constexpr int kU = kScanUnroll, kParts = ROW_THREADS / kSplitThreads;
   constexpr int VN = Row<T>::kPerVec;
   constexpr int NV = NVF + (ANY ? 2 : PARTIAL ? 1 : 0);
@@ -215,8 +220,7 @@ void actor_step_split_kernel(
     }
     return reg[j < LDS_VECS ? 0 : j - LDS_VECS];
   };
-  // this launch's tags: the counter was advanced by `laps` in front of the launch
-  const unsigned tag = exchange_tag(reinterpret_cast<const unsigned*>(ring + kRingWords), laps, row);
+  const unsigned first_tag = exchange_first_tag(tag_base, tag_word), tag = first_tag + unsigned(row / kRing);
   float my_gathered = 0.f;
   if constexpr (TOPK) {
     if (my_k >= 0) my_gathered = topk_gather_one<T>(a, logits + row * row_stride, vocab, my_id);
@@ -296,7 +300,8 @@ void actor_step_split_kernel(
     }
     bool any_gave_up = false;
     const SoftmaxAcc whole = split_collect<ROW_THREADS / kWave>(slot, tag + wait_tag_offset, tid, max_polls,
-                                                                reinterpret_cast<unsigned*>(ring + kRingWords), any_gave_up);
+                                                                reinterpret_cast<unsigned*>(ring + kRingWords),
+                                                                first_tag, any_gave_up);
     if constexpr (TOPK) {
       // the row's gathered logits, entry lane + 64 i from the workgroup that fetched it
       unsigned* status = reinterpret_cast<unsigned*>(ring + kRingWords);
@@ -305,10 +310,10 @@ void actor_step_split_kernel(
       for (int i = 0; i < kTopkPerLane; ++i) {
         const int k = tid + i * kWave;
         if (k < a.topk_k && !gave_up)
-          gave_up = !exchange_wait(topk_slot + k, tag + wait_tag_offset, max_polls, status, gathered.x[i]);
+          gave_up = !exchange_wait(topk_slot + k, tag + wait_tag_offset, max_polls, status, first_tag, gathered.x[i]);
       }
       const bool any_topk_gave_up = __any(gave_up);
-      if (any_topk_gave_up && !any_gave_up && tid == 0) exchange_report_give_up(status);
+      if (any_topk_gave_up && !any_gave_up && tid == 0) exchange_report_give_up(status, first_tag);
       any_gave_up = any_topk_gave_up;
     }
     float lse = 0.f, spx = 0.f, ent = 0.f, lp = 0.f;

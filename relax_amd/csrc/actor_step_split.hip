@@ -36,16 +36,16 @@
 
 namespace relax_amd {
 
-// the exchange ring and its status words
-static __device__ __align__(256) unsigned long long split_ring[kRingWords + kRingTailWords];
-// The logits at a token's top-K ids, gathered once per row: each workgroup of a row fetches its share of the K
-// scattered entries and publishes them here (one tagged word per entry, the ring's tags and status words), every
-// workgroup's first wave collects all K.  Gathered by each of the eight workgroups for itself, the K scattered lines
-// crossed the fabric eight times per row (3.4 GB on 65536 x 151936 rows with K = 64, a tenth of the step's traffic).
-static __device__ __align__(256) unsigned long long split_topk_ring[kTopkRingWords];
+// The exchange rings (1.5 MB each) and, of the same tags, those of the logits at a token's top-K ids (8 MB each).  The
+// logits are gathered once per row: each workgroup of a row fetches its share of the K scattered entries and publishes
+// them (one tagged word per entry), every workgroup's first wave collects all K.  Gathered by each of the eight workgroups
+// for itself, the K scattered lines crossed the fabric eight times per row (3.4 GB on 65536 x 151936 rows with K = 64, a
+// tenth of the step's traffic).
+static __device__ __align__(256) unsigned long long split_rings[exchange_array_words<kRingWords>()];
+static __device__ __align__(256) unsigned long long split_topk_rings[kExchangeRings * kTopkRingWords];
 
 namespace {
-ExchangeRingCache ring_cache, topk_ring_cache;
+ExchangeFamily split_family{"actor_step_split", {}};
 // relax_amd_set_exchange_wait: the bound of a workgroup's wait and an offset added to the tag it waits for
 std::atomic<unsigned> g_max_polls{kWaitPolls}, g_wait_tag_offset{0u};
 }  // namespace
@@ -53,12 +53,10 @@ std::atomic<unsigned> g_max_polls{kWaitPolls}, g_wait_tag_offset{0u};
 unsigned exchange_max_polls() { return g_max_polls.load(std::memory_order_relaxed); }
 unsigned exchange_wait_tag_offset() { return g_wait_tag_offset.load(std::memory_order_relaxed); }
 
-static int split_ring_of_device(unsigned long long** ring) {
-  return exchange_ring_of_device(ring_cache, reinterpret_cast<const void*>(&split_ring), "actor_step_split", ring);
-}
-static int split_topk_ring_of_device(unsigned long long** ring) {
-  return exchange_ring_of_device(topk_ring_cache, reinterpret_cast<const void*>(&split_topk_ring), "actor_step_split",
-                                 ring);
+int open_split_exchange(ExchangeLaunch& x, hipStream_t stream, int64_t n_rows, bool own_ring_only) {
+  return x.open<kRingWords>(split_family, reinterpret_cast<const void*>(&split_rings),
+                            reinterpret_cast<const void*>(&split_topk_rings), kTopkRingWords, stream,
+                            unsigned((n_rows + kRing - 1) / kRing), own_ring_only);
 }
 
 // Waves per SIMD the kernel is compiled for.  Long 16-bit rows without the top-K term run fastest with three (six
@@ -81,13 +79,13 @@ constexpr int split_waves_max() {
     if (a.topk_ids)                                                                                                   \
       hipLaunchKernelGGL((RELAX_AMD_SPLIT_KERNEL(WIDTH, NVF, PARTIAL, true)), grid, block, 0, stream, logits,        \
                          row_stride, vocab, n_rows, token_of_row, sample_ids, targets, inv_t * kLog2e, inv_t, a,     \
-                         grad_scale, log_prob, entropy, lse, spx, dlogits, d_stride, ring, topk_ring, laps,          \
-                         max_polls, tag_offset);                                                                      \
+                         grad_scale, log_prob, entropy, lse, spx, dlogits, d_stride, x.ring, x.extra,                 \
+                         x.base, x.word, max_polls, tag_offset);                                                      \
     else                                                                                                              \
       hipLaunchKernelGGL((RELAX_AMD_SPLIT_KERNEL(WIDTH, NVF, PARTIAL, false)), grid, block, 0, stream, logits,       \
                          row_stride, vocab, n_rows, token_of_row, sample_ids, targets, inv_t * kLog2e, inv_t, a,     \
-                         grad_scale, log_prob, entropy, lse, spx, dlogits, d_stride, ring, topk_ring, laps,          \
-                         max_polls, tag_offset);                                                                      \
+                         grad_scale, log_prob, entropy, lse, spx, dlogits, d_stride, x.ring, x.extra,                 \
+                         x.base, x.word, max_polls, tag_offset);                                                      \
     return check_launch("actor_step_split");                                                                          \
   }
 #define RELAX_AMD_SPLIT(NVF, PARTIAL) RELAX_AMD_SPLIT_ROW(1024, NVF, PARTIAL)
@@ -114,13 +112,13 @@ constexpr int split_lds_waves() {
       if constexpr (WITH_TOPK)                                                                                        \
         hipLaunchKernelGGL((RELAX_AMD_SPLIT_LDS_KERNEL(NVF, PARTIAL, true)), grid, block, 0, stream, logits,         \
                            row_stride, vocab, n_rows, token_of_row, sample_ids, targets, inv_t * kLog2e, inv_t, a,   \
-                           grad_scale, log_prob, entropy, lse, spx, dlogits, d_stride, ring, topk_ring, laps,        \
-                           max_polls, tag_offset);                                                                    \
+                           grad_scale, log_prob, entropy, lse, spx, dlogits, d_stride, x.ring, x.extra,               \
+                           x.base, x.word, max_polls, tag_offset);                                                    \
     } else {                                                                                                          \
       hipLaunchKernelGGL((RELAX_AMD_SPLIT_LDS_KERNEL(NVF, PARTIAL, false)), grid, block, 0, stream, logits,          \
                          row_stride, vocab, n_rows, token_of_row, sample_ids, targets, inv_t * kLog2e, inv_t, a,     \
-                         grad_scale, log_prob, entropy, lse, spx, dlogits, d_stride, ring, topk_ring, laps,          \
-                         max_polls, tag_offset);                                                                      \
+                         grad_scale, log_prob, entropy, lse, spx, dlogits, d_stride, x.ring, x.extra,                 \
+                         x.base, x.word, max_polls, tag_offset);                                                      \
     }                                                                                                                 \
     return check_launch("actor_step_split");                                                                          \
   }
@@ -160,15 +158,10 @@ int launch_actor_step_split(const T* logits, int64_t row_stride, int64_t vocab, 
           (full == 15 && partial) || (full == 16 && !partial)))
       return RELAX_AMD_EUNSUPPORTED;
   }
-  unsigned long long* ring = nullptr;
-  if (int rc = split_ring_of_device(&ring)) return rc;
-  unsigned long long* topk_ring = nullptr;
-  if (int rc = split_topk_ring_of_device(&topk_ring)) return rc;
-  const unsigned laps = unsigned((n_rows + kRing - 1) / kRing);
+  ExchangeLaunch x;
+  if (int rc = open_split_exchange(x, stream, n_rows, false)) return rc;
   const unsigned max_polls = exchange_max_polls();
   const unsigned tag_offset = exchange_wait_tag_offset();
-  hipLaunchKernelGGL(exchange_ring_advance_kernel<kRingWords>, dim3(1), dim3(256), 0, stream, ring, laps,
-                     topk_ring, kTopkRingWords);
   const dim3 grid(static_cast<unsigned>(n_rows * (width / kSplitThreads))), block(kSplitThreads);
   if constexpr (sizeof(T) == 2) {
     RELAX_AMD_SPLIT_ROW(512, 7, true)

@@ -13,49 +13,6 @@
 
 namespace relax_amd {
 
-// Exchange rings, one per stream: launches of different streams may overlap, and two of them on one ring would
-// overwrite each other's words.  The first kAnyRings streams of a process that come here get one each, per device; the
-// launches of later streams, and captured ones (whose replays may run beside the stream's own launches), are left to the
-// two-walk kernel.
-constexpr int kAnyRings = 4;
-constexpr size_t kAnyRingStride = kRingWords + kRingTailWords;
-static __device__ __align__(256) unsigned long long split_any_rings[kAnyRings * kAnyRingStride];
-
-namespace {
-ExchangeRingCache any_ring_cache;
-std::mutex any_streams_mutex;
-hipStream_t any_streams[ExchangeRingCache::kMaxDevices][kAnyRings];
-int any_streams_used[ExchangeRingCache::kMaxDevices];
-
-// the stream's ring, or null where it has none
-int any_ring_of_stream(hipStream_t stream, unsigned long long** ring) {
-  *ring = nullptr;
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
-    (void)hipGetLastError();
-    return RELAX_AMD_OK;
-  }
-  // a per-thread default stream is another stream in every thread under one handle
-  if (capture != hipStreamCaptureStatusNone || stream == hipStreamPerThread) return RELAX_AMD_OK;
-  unsigned long long* rings = nullptr;
-  if (int rc = exchange_ring_of_device(any_ring_cache, reinterpret_cast<const void*>(&split_any_rings),
-                                       "actor_step_split", &rings))
-    return rc;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return RELAX_AMD_OK;
-  std::lock_guard<std::mutex> lock(any_streams_mutex);
-  int& used = any_streams_used[dev];
-  int i = 0;
-  while (i < used && any_streams[dev][i] != stream) ++i;
-  if (i == used) {
-    if (used == kAnyRings) return RELAX_AMD_OK;
-    any_streams[dev][used++] = stream;
-  }
-  *ring = rings + size_t(i) * kAnyRingStride;
-  return RELAX_AMD_OK;
-}
-}  // namespace
-
 template <int NVF>
 constexpr int any_waves_min() {
   return NVF + 2 >= 15 ? 3 : 4;  // as split_waves_min()
@@ -68,14 +25,12 @@ constexpr int any_waves_max() {
 // One instantiation serves two row widths' worth of lengths (NVF .. NVF + 2 vectors per virtual thread).
 #define RELAX_AMD_SPLIT_ANY(WIDTH, NVF)                                                                               \
   if (width == WIDTH && nvec >= int64_t(NVF) * WIDTH && nvec <= int64_t(NVF + 2) * WIDTH) {                           \
-    hipLaunchKernelGGL(exchange_ring_advance_kernel<kRingWords>, dim3(1), dim3(256), 0, stream, ring, laps, nullptr,  \
-                       size_t(0));                                                                                    \
     hipLaunchKernelGGL((actor_step_split_kernel<T, NVF, false, false, WIDTH, any_waves_min<NVF>(),                    \
                                                 any_waves_max<NVF>(), 0, true>),                                      \
                        dim3(static_cast<unsigned>(n_rows * (width / kSplitThreads))), dim3(kSplitThreads), 0, stream, \
                        logits, row_stride, vocab, n_rows, token_of_row, sample_ids, targets, inv_t * kLog2e, inv_t,   \
-                       a, grad_scale, log_prob, entropy, lse, spx, dlogits, d_stride, ring, nullptr, laps,            \
-                       exchange_max_polls(), exchange_wait_tag_offset());                                             \
+                       a, grad_scale, log_prob, entropy, lse, spx, dlogits, d_stride, x.ring, nullptr, x.base,       \
+                       nullptr, exchange_max_polls(), exchange_wait_tag_offset());                                    \
     return check_launch("actor_step_split");                                                                          \
   }
 
@@ -92,10 +47,9 @@ int launch_actor_step_split_any(const T* logits, int64_t row_stride, int64_t voc
   // 16-bit rows of up to the 20 vectors per thread that the register file holds; the top-K term is left to the two-walk
   // kernel
   if (nvec < 4 * 512 || nvec > 20 * 1024 || a.topk_ids || n_rows * kSplit > 2147483647LL) return RELAX_AMD_EUNSUPPORTED;
-  unsigned long long* ring = nullptr;
-  if (int rc = any_ring_of_stream(stream, &ring)) return rc;
-  if (!ring) return RELAX_AMD_EUNSUPPORTED;
-  const unsigned laps = unsigned((n_rows + kRing - 1) / kRing);
+  // streams without an exchange ring of their own and captured launches are left to the two-walk kernel
+  ExchangeLaunch x;
+  if (int rc = open_split_exchange(x, stream, n_rows, true)) return rc;
   RELAX_AMD_SPLIT_ANY(512, 4)
   RELAX_AMD_SPLIT_ANY(512, 6)
   RELAX_AMD_SPLIT_ANY(512, 8)

@@ -35,7 +35,7 @@ constexpr int kKlSplitThreads = 128;
 constexpr int kKlSplit = kKlRowThreads / kKlSplitThreads;
 constexpr size_t kKlRingWords = size_t(kRing) * kKlSlotWords;
 
-static __device__ __align__(256) unsigned long long kl_split_ring[kKlRingWords + kRingTailWords];
+static __device__ __align__(256) unsigned long long kl_split_rings[exchange_array_words<kKlRingWords>()];
 
 // marks a raw vector as changed without touching it: what is unpacked from it afterwards is a new value to the
 // compiler, which would otherwise keep (and spill) the values unpacked earlier for the later uses
@@ -106,8 +106,8 @@ __global__ __launch_bounds__(kKlSplitThreads) __attribute__((amdgpu_waves_per_eu
 void reverse_kl_split_kernel(
     const T* __restrict__ student, const T* __restrict__ teacher, int64_t stride, int64_t vocab, int64_t n_rows,
     const float* __restrict__ g, float grad_scale, float* __restrict__ kl, float* __restrict__ lse_s,
-    float* __restrict__ lse_t, T* __restrict__ dstudent, unsigned long long* __restrict__ ring, unsigned laps,
-    unsigned max_polls, unsigned wait_tag_offset) {
+    float* __restrict__ lse_t, T* __restrict__ dstudent, unsigned long long* __restrict__ ring,
+    unsigned tag_base, const unsigned* __restrict__ tag_word, unsigned max_polls, unsigned wait_tag_offset) {
   constexpr int kU = kKlUnroll, ROW_THREADS = kKlRowThreads;
   constexpr int VN = Row<T>::kPerVec;
   constexpr int NV = NVF + (PARTIAL ? 1 : 0);
@@ -142,7 +142,7 @@ void reverse_kl_split_kernel(
   // teacher vector j of this thread
   auto teacher_vec = [&](int j) -> u32x4 { return j < LDS_VECS ? tlds[j < LDS_VECS ? j : 0][tid] : treg[j < LDS_VECS ? 0 : j - LDS_VECS]; };
   unsigned* status = reinterpret_cast<unsigned*>(ring + kKlRingWords);
-  const unsigned tag = exchange_tag(status, laps, row);
+  const unsigned first_tag = exchange_first_tag(tag_base, tag_word), tag = first_tag + unsigned(row / kRing);
   const float gt = g[row] * grad_scale;
 
   // the scan, pair by pair as the vectors arrive, in reverse_kl_step_kernel's order
@@ -191,11 +191,11 @@ void reverse_kl_split_kernel(
     // states in wave order
     __builtin_amdgcn_s_setprio(3);
     float lo = 0.f, hi = 0.f;
-    bool gave_up = !exchange_wait(slot + tid, tag + wait_tag_offset, max_polls, status, lo);
+    bool gave_up = !exchange_wait(slot + tid, tag + wait_tag_offset, max_polls, status, first_tag, lo);
     if (tid < kKlSlotWords - kWave && !gave_up)
-      gave_up = !exchange_wait(slot + kWave + tid, tag + wait_tag_offset, max_polls, status, hi);
+      gave_up = !exchange_wait(slot + kWave + tid, tag + wait_tag_offset, max_polls, status, first_tag, hi);
     const bool any_gave_up = __any(gave_up);
-    if (any_gave_up && tid == 0) exchange_report_give_up(status);
+    if (any_gave_up && tid == 0) exchange_report_give_up(status, first_tag);
     auto word = [&](int i) {  // word i of the slot, in every lane
       return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(i < kWave ? lo : hi), i & (kWave - 1)));
     };
@@ -254,7 +254,7 @@ void reverse_kl_split_kernel(
 }
 
 namespace {
-ExchangeRingCache kl_ring_cache;
+ExchangeFamily kl_family{"reverse_kl_split", {}};
 }
 
 // Long rows (12 and more vector positions per thread): three waves per SIMD, i.e. six workgroups per CU, each with
@@ -309,22 +309,19 @@ int launch_reverse_kl_split(const T* student, const T* teacher, int64_t stride, 
           (full == 16 && !partial) || (full == 12 && partial) || (full == 8 && !partial) || (full == 7 && partial) ||
           (full == 6 && partial)))
       return RELAX_AMD_EUNSUPPORTED;
-    unsigned long long* ring = nullptr;
-    if (int rc = exchange_ring_of_device(kl_ring_cache, reinterpret_cast<const void*>(&kl_split_ring),
-                                         "reverse_kl_split", &ring))
+    ExchangeLaunch x;
+    if (int rc = x.open<kKlRingWords>(kl_family, reinterpret_cast<const void*>(&kl_split_rings), nullptr, 0, stream,
+                                      unsigned((n_rows + kRing - 1) / kRing), false))
       return rc;
-    const unsigned laps = unsigned((n_rows + kRing - 1) / kRing);
     const unsigned max_polls = exchange_max_polls();
     const unsigned tag_offset = exchange_wait_tag_offset();
-    hipLaunchKernelGGL(exchange_ring_advance_kernel<kKlRingWords>, dim3(1), dim3(256), 0, stream, ring, laps,
-                       static_cast<unsigned long long*>(nullptr), size_t(0));
     const dim3 grid(static_cast<unsigned>(n_rows * kKlSplit)), block(kKlSplitThreads);
 #define RELAX_AMD_KL_SPLIT(NVF, PARTIAL)                                                                              \
   if (full == NVF && partial == PARTIAL) {                                                                            \
     hipLaunchKernelGGL((reverse_kl_split_kernel<T, NVF, PARTIAL, kl_split_lds_vecs<NVF>(), kl_split_waves_min<NVF>(), \
                                                 kl_split_waves_max<NVF>()>),                                          \
                        grid, block, 0, stream, student, teacher, stride, vocab, n_rows, g, grad_scale, kl, lse_s,    \
-                       lse_t, dstudent, ring, laps, max_polls, tag_offset);                                           \
+                       lse_t, dstudent, x.ring, x.base, x.word, max_polls, tag_offset);                                           \
     return check_launch("reverse_kl_split");                                                                          \
   }
     // 200064 / 201088 / 202048, 248320 / 250880, 256000, 262144 entries

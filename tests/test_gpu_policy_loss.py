@@ -7,6 +7,8 @@ element of magnitude ~2 cannot be represented more finely than 0.0078.  Token co
 
 BF16_ULP = 2.0 ** -7
 
+import threading
+
 import pytest
 import torch
 
@@ -2032,6 +2034,71 @@ def test_one_shot_step_on_rows_of_any_length_streams_capture_and_ring_laps():
         torch.cuda.synchronize()
         for a, b in zip(want, got):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("v", [16387, 32000])
+def test_one_shot_steps_of_two_threads_and_of_several_streams_stay_apart(v):
+    """Launches that two threads enqueue on one stream, and launches of more streams than own an exchange ring, without
+    a synchronization between them: every one of them gives the two-walk kernel's bits of its own inputs.  Row counts
+    of one lap each, so that the launches would have had equal tags if they were given the same counter."""
+    dev = require_gpu()
+    announce("one-shot steps, threads and streams", v)
+    steps = [_any_row_step(v, torch.bfloat16, 400 + i, 0, 7 + i, dev) for i in range(7)]
+    wants = [step("two_walk")[1] for step in steps]
+    torch.cuda.synchronize()
+    got = [[] for _ in steps]
+
+    def enqueue(i, stream, count):
+        with torch.cuda.stream(stream):
+            for _ in range(count):
+                name, out = steps[i]()
+                got[i].append(out)
+        return name
+
+    one = torch.cuda.default_stream()
+    threads = [threading.Thread(target=enqueue, args=(i, one, 30)) for i in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(5)]
+    for _ in range(4):
+        for i, stream in enumerate(streams):
+            name = enqueue(i + 2, stream, 1)
+            assert v == 16387 or name == "actor_step_split"  # the built row lengths keep it on any stream
+    torch.cuda.synchronize()
+    for i, outs in enumerate(got):
+        assert len(outs) == (30 if i < 2 else 4)
+        for out in outs:
+            for a, b in zip(wants[i], out):
+                assert torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("recorded", [1, 2])
+def test_captured_one_shot_steps_replayed_in_turn(recorded):
+    """Graphs that record the same kernel family share a ring: each replay takes tags of its own."""
+    dev = require_gpu()
+    announce("one-shot steps in several graphs")
+    steps = [_any_row_step(32000, torch.bfloat16, 4200 + 100 * i, 0, 3 + i, dev) for i in range(recorded)]
+    wants = [step("two_walk")[1] for step in steps]
+    graphs, outs = [], []
+    for step in steps:
+        step()
+        torch.cuda.synchronize()
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1]):
+            name, out = step()
+        assert name == "actor_step_split"
+        outs.append(out)
+    for _ in range(3):
+        for graph, step in zip(graphs, steps):
+            graph.replay()
+            step()
+        torch.cuda.synchronize()
+        for want, out in zip(wants, outs):
+            for a, b in zip(want, out):
+                assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("seed", range(16))
