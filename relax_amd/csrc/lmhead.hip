@@ -455,9 +455,11 @@ static void lm_plan_splits(int64_t row_blocks, LmGeom& g) {
   g.tasks.strip = lm_strip_height(row_blocks);
 }
 
-// floats of per-split softmax partials in the workspace (three per token and split)
+// Floats of per-split softmax partials in the workspace (three per token and split): room for whatever split count
+// lm_plan_splits() takes for this many tokens or fewer.  (Sized for the count alone it was 787 k floats at 256 tokens and
+// 769 k at 1000: a caller with one buffer for its largest chunk would have been written past by a shorter one.)
 static int64_t lm_partial_floats(int64_t n_tokens) {
-  return lm_max_splits((n_tokens + kLmTile - 1) / kLmTile) * 3 * n_tokens;
+  return std::max(kLmMaxTasks, (n_tokens + kLmTile - 1) / kLmTile) * kLmTile * 3;
 }
 
 static unsigned lm_grid(const LmGeom& g) { return lm_task_blocks(int64_t(g.tasks.rows) * g.tasks.cols); }
@@ -692,16 +694,11 @@ extern "C" int relax_amd_lmhead_live_rows(const void* rows, int64_t row_stride, 
   return check_launch("lmhead_live_gather");
 }
 
-static int64_t lm_live_partial_floats(int64_t max_tokens) {
-  const int64_t row_blocks = (max_tokens + kLmTile - 1) / kLmTile;
-  return std::max(kLmMaxTasks, row_blocks) * kLmTile * 3;
-}
-
 static int64_t lm_round4(int64_t x) { return (x + 3) / 4 * 4; }
 
 extern "C" int64_t relax_amd_lmhead_live_workspace_bytes(int64_t max_tokens, int64_t hidden_size) {
   if (max_tokens <= 0 || hidden_size <= 0) return 0;
-  return (lm_live_partial_floats(max_tokens) + 2 * lm_round4(max_tokens) +
+  return (lm_partial_floats(max_tokens) + 2 * lm_round4(max_tokens) +
           lm_live_dhidden_floats(max_tokens, hidden_size)) * int64_t(sizeof(float));
 }
 
@@ -751,7 +748,7 @@ extern "C" int relax_amd_lmhead_live_step(const void* plan, const void* picked, 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const LmLivePlan* live = static_cast<const LmLivePlan*>(plan);
   float* partial = static_cast<float*>(workspace);
-  float* x_target = partial + lm_live_partial_floats(max_tokens);
+  float* x_target = partial + lm_partial_floats(max_tokens);
   float* lse = x_target + lm_round4(max_tokens);
   float* dh_part = lse + lm_round4(max_tokens);
   uint16_t* l_t = static_cast<uint16_t*>(slab);

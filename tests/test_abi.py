@@ -112,6 +112,15 @@ def test_argument_validation_reports_errors_without_touching_the_gpu():
     assert L.relax_amd_whiten_partials(1) == 1 and L.relax_amd_whiten_partials(4097) == 2
 
 
+def test_lmhead_workspaces_of_a_longer_call_serve_every_shorter_one():
+    """``relax_amd_lmhead_logprob_fwd`` takes no workspace size: a buffer for the longest chunk has to do for the last one."""
+    from relax_amd._lib import lib
+
+    for size in (lib.relax_amd_lmhead_workspace_bytes, lambda n: lib.relax_amd_lmhead_live_workspace_bytes(n, 4096)):
+        have = [size(n) for n in list(range(1, 9000)) + list(range(9000, 300000, 97))]
+        assert have[0] > 0 and all(a <= b for a, b in zip(have, have[1:]))
+
+
 def test_product_refuses_cpu_tensors():
     import relax_amd
     from relax_amd import ppo_utils
