@@ -530,6 +530,26 @@ def test_token_means_in_one_launch_vs_float64(n):
     assert ops.token_mean(x[:0].to(dev), x[:0].to(dev))[0].item() == 0
 
 
+@pytest.mark.parametrize("n", [262144, 262145, 300001])
+def test_token_mean_leaves_the_single_workgroup_where_it_loses(n, monkeypatch):
+    """Means on either side of the size up to which one workgroup is used, by the bound of the test above."""
+    from relax_amd import ops
+    from relax_amd._lib import lib
+
+    dev = require_gpu()
+    announce("token mean, many tokens", n)
+    calls, single = [], lib.relax_amd_token_mean
+    monkeypatch.setattr(lib, "relax_amd_token_mean", lambda *a: calls.append(n) or single(*a))
+    g = torch.Generator().manual_seed(n)
+    x, mask = torch.randn(n, generator=g), (torch.rand(n, generator=g) > 0.4).float()
+    mean, got_den = ops.token_mean(x.to(dev), mask.to(dev))
+    den = mask.double().sum().item()
+    want = ((x * mask).double().sum() / den).item()
+    assert got_den.dtype == torch.float64 and got_den.item() == den
+    assert abs(mean.item() - want) <= 2.0 ** -23 * abs(want) + 1e-12
+    assert len(calls) == (n <= ops.TOKEN_MEAN_SUM_MAX)
+
+
 def test_opd_token_mean_literal(literals):
     from relax_amd.opd_utils import compute_opd_kl, reduce_opd_loss
 
