@@ -13,7 +13,7 @@ import threading
 import torch
 
 _SLOTS = 8
-_CAPACITY = 1 << 14  # int64 elements per slot
+CAPACITY = 1 << 16  # int64 elements per slot (512 KB): the packing table of 4096 samples with five fields
 
 _local = threading.local()
 
@@ -22,7 +22,7 @@ class _Slot:
     __slots__ = ("buf", "event")
 
     def __init__(self):
-        self.buf = torch.empty(_CAPACITY, dtype=torch.int64, pin_memory=True)
+        self.buf = torch.empty(CAPACITY, dtype=torch.int64, pin_memory=True)
         self.event = None
 
 
@@ -31,7 +31,7 @@ def upload_int64(values, device) -> torch.Tensor:
     host = values if isinstance(values, torch.Tensor) else torch.tensor(values, dtype=torch.int64)
     host = host.to(torch.int64).reshape(-1)
     n = host.numel()
-    if n > _CAPACITY or n == 0:
+    if n > CAPACITY or n == 0:
         return host.to(device)
     ring = getattr(_local, "ring", None)
     if ring is None:

@@ -25,7 +25,7 @@ import torch
 
 from . import ops
 from ._lib import METRIC_SLOTS
-from ._staging import upload_int64
+from ._staging import CAPACITY as STAGING_CAPACITY, upload_int64
 from .cp_utils import (MaskedSampleReduce, PerSampleDivisorReducer, get_cp_local_num_tokens,
                        get_sum_of_sample_mean, sample_denominators)
 
@@ -167,7 +167,10 @@ class PackedLayout:
     def _pack(self, device, n_rows, unconcat_tokens, begins, sft, cu, need_inverse, fields, denom_of) -> bool:
         """The one-launch form; False where the batch is not of that form."""
         b, lengths = self.n_samples, self.response_lengths
-        if self.n_tokens == 0 or not self.rows_once or len(unconcat_tokens) != b or b > 4096:
+        if self.n_tokens == 0 or not self.rows_once or len(unconcat_tokens) != b:
+            return False
+        # a table larger than a staging slot would be copied from pageable memory, which waits for all queued launches
+        if 2 * b + 1 + b * (7 + sum(v is not None for v in fields.values())) > STAGING_CAPACITY:
             return False
         if torch.cuda.is_current_stream_capturing():  # addresses of this batch's tensors do not belong in a graph
             return False

@@ -767,6 +767,40 @@ def test_packed_batch_equals_its_pieces(tot, resp, extra):
         assert torch.equal(lay.fields["old"], want) and lay.denom is None
 
 
+@pytest.mark.parametrize("b", [1171, 4096, 5000])
+def test_packing_tables_of_many_samples_travel_through_the_pinned_staging(b, monkeypatch):
+    """A table larger than a staging slot would be a pageable copy, on which the host waits for every queued launch: the
+    slots hold the table of 4096 samples, and larger batches go piece by piece, with the same result."""
+    from relax_amd import _staging, loss
+    from relax_amd.cp_utils import sample_denominators
+
+    dev = require_gpu()
+    announce("packing table", b)
+    uploads, upload = [], loss.upload_int64
+    monkeypatch.setattr(loss, "upload_int64", lambda values, device: uploads.append(len(values)) or upload(values, device))
+    g = torch.Generator().manual_seed(b)
+    resp = torch.randint(1, 4, (b,), generator=g).tolist()
+    tot = [r + 1 for r in resp]
+
+    def pieces(x, lens):
+        return [t.clone() for t in torch.split(x.to(dev), lens)]
+
+    toks = pieces(torch.randint(0, 1000, (sum(tot),), generator=g), tot)
+    masks = pieces((torch.rand(sum(resp), generator=g) > 0.5).float(), resp)
+    fields = dict({k: pieces(torch.randn(sum(resp), generator=g), resp) for k in ("old", "rollout", "ref", "advantages")},
+                  masks=masks)
+    lay = loss.PackedLayout(dev, sum(tot), toks, tot, resp, True, fields=fields, denom_of="masks")
+    assert (lay.denom is not None) == (b <= 4096)
+    other = loss.PackedLayout(dev, sum(tot), [t.int() for t in toks], tot, resp, True, fields=fields)
+    for name in ("row_ids", "sample_ids", "token_of_row", "targets"):
+        assert torch.equal(getattr(lay, name), getattr(other, name)), name
+    for name in fields:
+        assert torch.equal(lay.fields[name], other.fields[name]), name
+    if b <= 4096:
+        assert torch.equal(lay.denom, sample_denominators(masks, other))
+    assert uploads and max(uploads) <= _staging.CAPACITY
+
+
 def test_full_size_packed_varlen_gspo_and_cispo_properties():
     """Packed variable-length batch at the benchmark's vocabulary (8 sequences, 2k-6k tokens here to bound the test's
     memory; the kernels are per-row): sequence-level GSPO through the two-launch path and token-level CISPO through the
