@@ -668,7 +668,9 @@ int relax_amd_lmhead_dlogits_from_logits_t(void* logits_t, int64_t n_tokens, int
  *      gradient rows d_rows[row] of the live tokens (others untouched; NULL: not wanted) and d_weight (_BF16 / _F32:
  *      written, zeros where nothing is live; _F32_ACCUMULATE: added to; NULL: not wanted).  slab: bf16
  *      [>= ceil128(vocab), slab_stride >= ceil128(max_tokens)], rows >= vocab zero, overwritten.  workspace: 16-byte
- *      aligned, relax_amd_lmhead_live_workspace_bytes(max_tokens, hidden_size).
+ *      aligned, relax_amd_lmhead_live_step_workspace_bytes(max_tokens, hidden_size, vocab), most of it fp32 partial
+ *      products of the hidden gradient; relax_amd_lmhead_live_workspace_bytes(max_tokens, hidden_size) is enough for any
+ *      vocabulary.
  */
 int64_t relax_amd_lmhead_live_plan_bytes(int64_t n_tokens, int64_t slab_tokens);
 int relax_amd_lmhead_live_rows(const void* rows, int64_t row_stride, int64_t hidden_size, int64_t vocab,
@@ -677,6 +679,7 @@ int relax_amd_lmhead_live_rows(const void* rows, int64_t row_stride, int64_t hid
                                int32_t* token_map, void* picked, int64_t* picked_targets, float* g_lp,
                                int32_t* row_map, void* stream);
 int64_t relax_amd_lmhead_live_workspace_bytes(int64_t max_tokens, int64_t hidden_size);
+int64_t relax_amd_lmhead_live_step_workspace_bytes(int64_t max_tokens, int64_t hidden_size, int64_t vocab);
 int relax_amd_lmhead_live_step(const void* plan, const void* picked, const void* weight, int64_t w_stride,
                                int64_t max_tokens, int64_t hidden_size, int64_t vocab, const int64_t* picked_targets,
                                const float* g_lp, const int32_t* token_map, const int32_t* row_map,

@@ -125,6 +125,7 @@ SIGNATURES = {
     "relax_amd_lmhead_live_rows": (
         C.c_int, [_vp, _i64, _i64, _i64, _vp, _vp, _vp, _f32, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "relax_amd_lmhead_live_workspace_bytes": (_i64, [_i64, _i64]),
+    "relax_amd_lmhead_live_step_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "relax_amd_lmhead_live_step": (
         C.c_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _f32, _vp, _i64, _i64, _vp, _i64, _vp, _vp,
                   _i64, _vp, _i64, C.c_int, _vp]),

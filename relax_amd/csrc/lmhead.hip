@@ -696,10 +696,18 @@ extern "C" int relax_amd_lmhead_live_rows(const void* rows, int64_t row_stride, 
 
 static int64_t lm_round4(int64_t x) { return (x + 3) / 4 * 4; }
 
-extern "C" int64_t relax_amd_lmhead_live_workspace_bytes(int64_t max_tokens, int64_t hidden_size) {
+static int64_t lm_live_workspace_bytes(int64_t max_tokens, int64_t hidden_size, int64_t vocab) {
   if (max_tokens <= 0 || hidden_size <= 0) return 0;
   return (lm_partial_floats(max_tokens) + 2 * lm_round4(max_tokens) +
-          lm_live_dhidden_floats(max_tokens, hidden_size)) * int64_t(sizeof(float));
+          lm_live_dhidden_floats(max_tokens, hidden_size, vocab)) * int64_t(sizeof(float));
+}
+
+extern "C" int64_t relax_amd_lmhead_live_workspace_bytes(int64_t max_tokens, int64_t hidden_size) {
+  return lm_live_workspace_bytes(max_tokens, hidden_size, 0);
+}
+
+extern "C" int64_t relax_amd_lmhead_live_step_workspace_bytes(int64_t max_tokens, int64_t hidden_size, int64_t vocab) {
+  return vocab <= 0 ? 0 : lm_live_workspace_bytes(max_tokens, hidden_size, vocab);
 }
 
 extern "C" int relax_amd_lmhead_live_step(const void* plan, const void* picked, const void* weight, int64_t w_stride,
@@ -717,7 +725,7 @@ extern "C" int relax_amd_lmhead_live_step(const void* plan, const void* picked, 
     return rc;
   if (!plan || !picked_targets || !g_lp || !token_map || !row_map || !slab || !workspace || !log_prob ||
       !(inv_temperature > 0.f) || !aligned16(workspace) ||
-      workspace_bytes < relax_amd_lmhead_live_workspace_bytes(max_tokens, hidden_size)) {
+      workspace_bytes < lm_live_workspace_bytes(max_tokens, hidden_size, vocab)) {
     set_error("%s: NULL argument, non-positive inv_temperature or short workspace", what);
     return RELAX_AMD_EINVAL;
   }

@@ -637,9 +637,26 @@ extern "C" int relax_amd_lmhead_dweight(const void* d_t, int64_t d_stride, const
 
 // ---- the products of a live slab
 
-int64_t relax_amd::lm_live_dhidden_floats(int64_t max_tokens, int64_t hidden_size) {
+// Row blocks times splits of the contraction that a slab's plan can name at most (lmhead_live_plan_kernel takes the split
+// of least cost for the row blocks that turn out to be live: the maximum over those).  The partial products are sized and
+// the launch is laid out for it: 67 MB instead of 268 MB at 200 tokens of H = 4096, V = 151936, where every allowed split
+// had been provided for.
+static int64_t live_dhidden_row_splits(int64_t max_tokens, int64_t hidden_size, int64_t vocab) {
+  const int64_t rows = (max_tokens + kLmTile - 1) / kLmTile;
+  int64_t most = 1;
+  for (int64_t r = 1; r <= rows; ++r) {
+    GemmTiling t = gemm_tiling(r * kLmTile, hidden_size, ceil128(vocab));
+    gemm_plan_splits(gemm_max_splits(r), t);
+    most = std::max(most, r * t.splits);
+  }
+  return most;
+}
+
+int64_t relax_amd::lm_live_dhidden_floats(int64_t max_tokens, int64_t hidden_size, int64_t vocab) {
   const int64_t rows = (max_tokens + kLmTile - 1) / kLmTile, cols = (hidden_size + kLmTile - 1) / kLmTile;
-  return std::max<int64_t>(64, rows * gemm_max_splits(rows)) * cols * kLmTile * kLmTile;
+  const int64_t row_splits = vocab > 0 ? live_dhidden_row_splits(max_tokens, hidden_size, vocab)
+                                       : std::max<int64_t>(64, rows * gemm_max_splits(rows));  // of any vocabulary
+  return row_splits * cols * kLmTile * kLmTile;
 }
 
 int relax_amd::lm_live_dhidden(const void* d_t, int64_t d_stride, const void* weight, int64_t w_stride,
@@ -649,7 +666,7 @@ int relax_amd::lm_live_dhidden(const void* d_t, int64_t d_stride, const void* we
   const GemmOperand B = {static_cast<const uint16_t*>(weight), w_stride, hidden_size, vocab};
   const GemmTiling t = gemm_tiling(max_tokens, hidden_size, ceil128(vocab));
   const int64_t part_stride = int64_t(t.tiles.cols) * kLmTile;
-  const int64_t most = std::max<int64_t>(64, t.tiles.rows * gemm_max_splits(t.tiles.rows)) * t.tiles.cols;
+  const int64_t most = live_dhidden_row_splits(max_tokens, hidden_size, vocab) * t.tiles.cols;
   hipLaunchKernelGGL((lmhead_gemm_kernel<true, true, kGemmOutF32, false, kGemmLiveRows>), dim3(lm_task_blocks(most)),
                      dim3(kLmThreads), 0, s, A, B, part, part_stride, int64_t(0), int64_t(0), part_stride, t, live);
   if (int rc = check_launch("lmhead_dhidden")) return rc;

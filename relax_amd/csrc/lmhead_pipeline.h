@@ -468,7 +468,8 @@ struct LmSlabWriter {
 int lm_live_dhidden(const void* d_t, int64_t d_stride, const void* weight, int64_t w_stride, int64_t max_tokens,
                     int64_t hidden_size, int64_t vocab, const LmLivePlan* live, float* part, const int32_t* row_map,
                     void* d_rows, int64_t dr_stride, hipStream_t s);
-int64_t lm_live_dhidden_floats(int64_t max_tokens, int64_t hidden_size);
+// floats of dhidden's partial products (vocab 0: enough for any vocabulary)
+int64_t lm_live_dhidden_floats(int64_t max_tokens, int64_t hidden_size, int64_t vocab);
 int lm_live_dweight(const void* d_t, int64_t d_stride, const void* hidden, int64_t h_stride, int64_t max_tokens,
                     int64_t hidden_size, int64_t vocab, const LmLivePlan* live, void* d_weight, int64_t dw_stride,
                     int out_mode, hipStream_t s);

@@ -365,7 +365,7 @@ class _LMHeadLiveStep(torch.autograd.Function):
         d_rows = torch.zeros(rows.shape, dtype=torch.bfloat16, device=dev) if need_h else None
         d_weight = empty(torch.bfloat16 if single else torch.float32, v, h) if need_w else None
         slab = alloc_slab(v, min(n, slab_tokens), dev, columns=False)
-        ws_bytes = lib.relax_amd_lmhead_live_workspace_bytes(min(n, slab_tokens), h)
+        ws_bytes = lib.relax_amd_lmhead_live_step_workspace_bytes(min(n, slab_tokens), h, v)
         ws = empty(torch.uint8, ws_bytes)
         with ops._timed("lmhead_live_step"):
             check(lib.relax_amd_lmhead_live_rows(

@@ -121,6 +121,30 @@ def test_lmhead_workspaces_of_a_longer_call_serve_every_shorter_one():
         assert have[0] > 0 and all(a <= b for a, b in zip(have, have[1:]))
 
 
+@pytest.mark.parametrize("n,h,v", [(1, 128, 700), (200, 4096, 151936), (300, 2048, 32000), (4400, 128, 300),
+                                   (5200, 5120, 102400), (8192, 4096, 151936)])
+def test_live_step_workspace_holds_the_largest_plan_and_no_more(n, h, v):
+    """The partial products of the live LM-head step: row blocks x splits of the contraction at their maximum over the
+    counts of live tokens, each split the cheapest one by the documented cost (rounds of 256 workgroups, steps of 128
+    contraction elements, the partials' traffic)."""
+    from relax_amd._lib import lib
+
+    def ceil(a, b):
+        return -(-a // b)
+
+    cols, steps, most = ceil(h, 256), ceil(v, 128), 0
+    for rows in range(1, ceil(n, 256) + 1):
+        limit = min(4 if rows > 16 else 64 // rows, steps)
+        tiles = rows * cols
+        split = min(range(1, limit + 1), key=lambda s: ceil(tiles * s, 256) * (ceil(steps, s) + 3)
+                    + (s * tiles // 32 + 6 if s > 1 else 0))
+        most = max(most, rows * ceil(steps, ceil(steps, split)))
+    others = max(1024, ceil(n, 256)) * 256 * 3 + 2 * ceil(n, 4) * 4
+    size = lib.relax_amd_lmhead_live_step_workspace_bytes(n, h, v)
+    assert size == 4 * (others + most * cols * 256 * 256)
+    assert size <= lib.relax_amd_lmhead_live_workspace_bytes(n, h)
+
+
 def test_product_refuses_cpu_tensors():
     import relax_amd
     from relax_amd import ppo_utils
