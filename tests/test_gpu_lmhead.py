@@ -643,6 +643,64 @@ def test_sft_losses_plain_and_with_deferred_lm_head_vs_oracle():
         relax_amd.sft_loss_function_chunked(args, dbatch, hd, None, lm_head_forward=lambda x: x)
 
 
+@pytest.mark.parametrize("mode", ["per_token", "mask_sums", "int_masks"])
+def test_deferred_lm_head_sft_step_weights_its_tokens_as_the_reducer_does(mode):
+    """The weights the step takes without a reducer (token sum; the caller's per-sample divisors, one of them below one;
+    integer masks): loss and both gradients against the oracle's composition, by itself and under the scaling of
+    ``loss_function``, to the bounds of the test above."""
+    import relax_amd
+    from oracle import reducers as R
+
+    dev = require_gpu()
+    announce("sft lm head weights", mode)
+    g = torch.Generator().manual_seed(11)
+    tot, resp, h, v = [9, 14, 6, 5], [9, 6, 5, 2], 128, 300
+    hid = torch.randn(1, sum(tot), h, generator=g).bfloat16()
+    w = (torch.randn(v, h, generator=g) * 0.1).bfloat16()
+    toks = [torch.randint(0, v, (n,), generator=g) for n in tot]
+    masks = [(torch.rand(r, generator=g) > 0.3) for r in resp]
+    masks = [m.long() if mode == "int_masks" else m.float() for m in masks]
+    sums = torch.tensor([7.0, 0.25, 19.0, 2.0]) if mode == "mask_sums" else None
+    per_token = mode == "per_token"
+    hc, wc = hid.clone().requires_grad_(), w.clone().requires_grad_()
+    lps = []
+    for (b, e, _), tk, r in zip(P.response_row_ranges(tot, resp), toks, resp):
+        tg = F.pad(tk[1:], (0, 1), value=0) if r == tk.numel() else tk[-r:]
+        lps.append(P.lm_head_log_probs(hc[0, b:e], wc, tg, temperature=0.9, sub_chunk=4))
+    want = -R.make_reducer(resp, masks, per_token, sums)(torch.cat(lps))
+    want.backward()
+    # 2e-3 per sample mean; a token sum, or a divisor smaller than the sample's mask sum, multiplies it accordingly
+    weight_sum = sum(m.sum().item() / (1.0 if per_token else max(m.sum().item() if sums is None else sums[i].item(), 1.0))
+                     for i, m in enumerate(masks))
+    args = P.make_args(loss_type="sft", sft_chunked_logits=True, rollout_temperature=0.9, global_batch_size=3,
+                       calculate_per_token_loss=per_token)
+    batch = dict(unconcat_tokens=[x.to(dev) for x in toks], total_lengths=tot, response_lengths=resp,
+                 loss_masks=[m.to(dev) for m in masks])
+    if sums is not None:
+        batch["sample_index_mask_sums"] = sums.to(dev)
+    for scaled in (False, True):
+        hd, wd = hid.to(dev).requires_grad_(), w.to(dev).requires_grad_()
+        factor = 1.0
+        if scaled:
+            loss, normalizer, log = relax_amd.loss_function(args, batch, 2, hd, lm_head_forward=wd)
+            factor = 1.0 if per_token else 2 / 3
+            assert int(normalizer) == (int(sum(m.sum() for m in masks)) if per_token else 1)
+            reported = log["values"][1]
+        else:
+            loss, log = relax_amd.sft_loss_function_chunked(args, batch, hd, None, lm_head_forward=wd)
+            reported = log["loss"]
+        loss.backward()
+        assert abs(loss.item() - want.item() * factor) < 2e-3 * max(1.0, weight_sum)
+        assert abs(reported.item() - want.item()) < 2e-3 * max(1.0, weight_sum)
+        for got, ref in ((hd.grad, hc.grad), (wd.grad, wc.grad)):
+            scale = ref.float().abs().max().item()
+            torch.testing.assert_close(got.float().cpu(), ref.float() * factor, atol=max(5e-3, 2 * BF16_ULP * scale),
+                                       rtol=2 * BF16_ULP)
+            # over a whole gradient: the oracle's logits are rounded to bf16 (up to 8e-3 of a probability where |x| < 4),
+            # the logits gradient and the result to half an ulp each
+            assert (got.float().cpu() - ref.float() * factor).norm() < (8e-3 + BF16_ULP) * (ref.float() * factor).norm()
+
+
 def test_model_forward_under_bypass_feeds_the_fused_loss_end_to_end():
     """A small model run under ``bypass_output_layer`` returns hidden states; ``loss_function`` with the yielded handle
     gives the loss and the gradients (LM-head weight and the layers below it) of the same model run normally with
