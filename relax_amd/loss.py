@@ -1403,7 +1403,9 @@ def compute_advantages_and_returns(args: Namespace, rollout_data: dict) -> None:
                 token_rewards.append(k)
         else:
             flat = torch.cat(kl[:n_rewarded]) * (-kl_coef) if n_rewarded else torch.zeros(0, device=dev)
-            last = upload_int64([e - 1 for e in itertools.accumulate(lens)], dev)
+            last = [e - 1 for e in itertools.accumulate(lens)]
+            # (the critic's values decide where the scan runs: the log-probs that only lend their shapes may lie on the host)
+            last = upload_int64(last, dev) if flat.is_cuda else torch.tensor(last, dtype=torch.int64)
             flat[last] += torch.tensor(rewards[:n_rewarded], dtype=flat.dtype, device=dev)
             token_rewards = list(torch.split(flat, lens))
         advantages, returns = get_advantages_and_returns_batch(

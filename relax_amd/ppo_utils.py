@@ -225,7 +225,7 @@ def broadcast_rewards(rewards, like):
     views in the shapes of ``like``.  One launch; a rollout batch has hundreds of samples, so nothing is done per sample
     that a whole-batch call can do."""
     lens = [x.numel() for x in like]
-    dev = like[0].device
+    dev = ops._need_gpu(like[0])
     flat = ops.broadcast_per_sample(rewards.to(dev).float(), upload_int64([0] + list(_accumulate(lens)), dev), sum(lens))
     return flat, [p if x.dim() == 1 else p.reshape(x.shape) for p, x in zip(torch.split(flat, lens), like)]
 

@@ -160,6 +160,23 @@ def test_product_refuses_cpu_tensors():
         ppo_utils.compute_approx_kl(torch.zeros(2), torch.zeros(2), "unsupported")
 
 
+@pytest.mark.parametrize("estimator", ["grpo", "rloo", "ppo", "reinforce_plus_plus"])
+def test_advantages_refuse_cpu_tensors(estimator):
+    from types import SimpleNamespace
+
+    import relax_amd
+    from relax_amd import ppo_utils
+
+    lens = [3, 2]
+    data = dict(log_probs=[torch.zeros(n) for n in lens], values=[torch.zeros(n) for n in lens], rewards=[1.0, 2.0],
+                loss_masks=[torch.ones(n) for n in lens], response_lengths=lens, total_lengths=lens)
+    args = SimpleNamespace(advantage_estimator=estimator, kl_coef=0.0, gamma=1.0, lambd=0.9, normalize_advantages=False)
+    with pytest.raises(RuntimeError, match="no CPU fallback"):
+        relax_amd.compute_advantages_and_returns(args, data)
+    with pytest.raises(RuntimeError, match="no CPU fallback"):
+        ppo_utils.get_grpo_returns(torch.ones(2), data["log_probs"])
+
+
 def test_host_index_arithmetic_matches_oracle_bruteforce():
     from oracle.policy import response_row_ranges
     from relax_amd.loss import response_row_begins

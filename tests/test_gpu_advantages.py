@@ -102,6 +102,25 @@ def test_group_rewards_across_staging_rounds(n, dtype, mode):
     torch.testing.assert_close(got.cpu().double(), want, rtol=0, atol=8 * (n / 7 + 1) * eps, equal_nan=True)
 
 
+def test_ppo_takes_log_probs_that_lie_on_the_host():
+    """Without a KL coefficient the log-probs only lend their shapes; the scan runs where the values lie."""
+    import relax_amd
+
+    dev = require_gpu()
+    announce("ppo, log-probs on the host")
+    lens = [5, 1, 130]
+    values = [torch.randn(n, device=dev) for n in lens]
+    args = SimpleNamespace(advantage_estimator="ppo", kl_coef=0.0, gamma=0.99, lambd=0.95, normalize_advantages=False)
+    results = []
+    for where in (dev, torch.device("cpu")):
+        data = dict(log_probs=[torch.randn(n, device=where) for n in lens], values=values, rewards=[0.5, -1.0, 2.0],
+                    response_lengths=lens, total_lengths=lens, loss_masks=[torch.ones(n, device=dev) for n in lens])
+        relax_amd.compute_advantages_and_returns(args, data)
+        results.append(list(data["advantages"]) + list(data["returns"]))
+    for a, b in zip(*results):
+        assert b.is_cuda and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("kl_coef", [0.0, 0.05])
 def test_ppo_token_rewards_of_a_batch_equal_the_per_sample_ones(kl_coef):
     """Advantages and returns of the whole-batch token rewards against GAE on rewards built sample by sample."""
