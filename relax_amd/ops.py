@@ -573,6 +573,8 @@ def group_rewards(rewards, group_index, mode: str):
 
 def broadcast_per_sample(per_sample, cu_resp, n_tokens: int):
     dev = _need_gpu(per_sample, cu_resp)
+    if per_sample.numel() < cu_resp.numel() - 1:
+        raise ValueError(f"{per_sample.numel()} per-sample values for {cu_resp.numel() - 1} samples")
     out = torch.empty(n_tokens, dtype=torch.float32, device=dev)
     check(lib.relax_amd_broadcast_per_sample(_p(_f32(per_sample)), _p(cu_resp), cu_resp.numel() - 1, _p(out),
                                              _stream()))

@@ -102,6 +102,21 @@ def test_group_rewards_across_staging_rounds(n, dtype, mode):
     torch.testing.assert_close(got.cpu().double(), want, rtol=0, atol=8 * (n / 7 + 1) * eps, equal_nan=True)
 
 
+def test_fewer_rewards_than_responses_are_refused():
+    """The broadcast reads a value per sample: too few of them are an error on the host, not a read past their end."""
+    import relax_amd
+    from relax_amd.ppo_utils import get_grpo_returns
+
+    dev = require_gpu()
+    announce("fewer rewards than responses")
+    like = [torch.zeros(n, device=dev) for n in (3, 2, 4)]
+    with pytest.raises(ValueError, match="2 per-sample values for 3 samples"):
+        get_grpo_returns(torch.ones(2, device=dev), like)
+    args = SimpleNamespace(advantage_estimator="grpo", kl_coef=0.0, normalize_advantages=False)
+    with pytest.raises(ValueError, match="2 per-sample values for 3 samples"):
+        relax_amd.compute_advantages_and_returns(args, dict(log_probs=like, rewards=[1.0, 2.0]))
+
+
 def test_ppo_takes_log_probs_that_lie_on_the_host():
     """Without a KL coefficient the log-probs only lend their shapes; the scan runs where the values lie."""
     import relax_amd
