@@ -503,9 +503,9 @@ int relax_amd_topk_rows(const void* logits, int dtype, int64_t n_tokens, int64_t
  * get_log_probs_and_entropy(..., with_topk=True) computes per sample (relax/backends/megatron/loss.py:373-446: the
  * log-probs / entropy of the response tokens and torch.topk of the same logits rows).  Arguments as in those two
  * functions; log_prob / entropy / lse / spx are bit-identical to relax_amd_logprob_entropy_fwd's, values / indices
- * follow relax_amd_topk_rows' contract (the selection does not depend on the temperature).  Rows that are not whole
- * 16-byte vectors in groups of eight, or too short for the forward scan's 1024-thread workgroups (fewer than 7168
- * vectors), run the two passes one after the other.
+ * follow relax_amd_topk_rows' contract (the selection does not depend on the temperature).  One read serves rows of
+ * 7168 .. 40959 whole 16-byte vectors (the forward scan's 1024-thread workgroups; up to 36863 where elements follow the
+ * last whole vector), at any address; others run the two passes one after the other.
  */
 int relax_amd_logprob_entropy_topk_fwd(const void* logits, int dtype, int64_t n_tokens, int64_t vocab,
                                        int64_t row_stride, const int32_t* row_ids, const int64_t* targets,
@@ -534,9 +534,11 @@ int relax_amd_logprob_entropy_topk_fwd(const void* logits, int dtype, int64_t n_
  * results bit for bit: one-shot workgroups that share each row (one read and one write of HBM per row; 16-bit rows of
  * 28680 .. 32768, 49160 .. 53248, 57352 .. 65536, 100352 .. 163840, 196616 .. 204800 and 245768 .. 262144 entries
  * (the last two ranges keep part of the row in LDS), fp32 rows of 28676 .. 32768, 49156 .. 53248,
- * 61444 .. 65536 and, part of the row in LDS, 100352 .. 163840 and 245764 .. 249856 entries, in the built shapes: the default where built, see
- * relax_amd_set_kernel_choice for the ring in device memory it exchanges partial sums through), a persistent
- * register-resident one (the same traffic, the same shapes) and a two-walk one for everything
+ * 61444 .. 65536 and, part of the row in LDS, 100352 .. 163840 and 245764 .. 249856 entries, in the built shapes, rows and
+ * strides of whole 16-byte vectors; without the top-K term also 16-bit rows of any length from 16384 to 163847 at any
+ * address, on the first four streams of a GPU that make such calls and outside graph capture: the default where built, see
+ * relax_amd_set_kernel_choice for the rings in device memory they exchange partial sums through), a persistent
+ * register-resident one (the same traffic, the built shapes) and a two-walk one for everything
  * else; relax_amd_set_kernel_choice(RELAX_AMD_KERNEL_RESIDENT / RELAX_AMD_KERNEL_TWO_WALK) forces the second / third.
  */
 int relax_amd_actor_step_fused(const void* logits, int dtype, int64_t n_rows, int64_t vocab, int64_t row_stride,

@@ -25,7 +25,7 @@ FLAGS = [
     "-fno-gpu-rdc",
     "-Wall",
     "-Wno-unused-function",
-    # packed-fp32 VALU forms are kept off on this hardware pool
+    # packed-fp32 VALU forms are kept off: some of them have given wrong results on this card
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     f"-I{INCLUDE}",
     f"-I{CSRC}",
