@@ -120,6 +120,12 @@ const char* relax_amd_last_kernel(void);
  * Process-wide, read at each launch.  No counterpart in the reference.
  */
 int relax_amd_set_exchange_wait(int max_polls, int wait_tag_offset);
+/*
+ * For tests of the rings' clearing, which precedes the launch that would need a 33rd bit of tag: counts the tags up to
+ * `used` of the current GPU's rings as handed out.  A ring that is further on stays where it is, so no tag comes twice.
+ * The GPU must be idle.  No counterpart in the reference.
+ */
+int relax_amd_advance_exchange_tags(uint32_t used);
 
 /*
  * Target-token log-prob and full-vocab entropy of each row, one streaming

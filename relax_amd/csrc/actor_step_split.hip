@@ -53,6 +53,8 @@ std::atomic<unsigned> g_max_polls{kWaitPolls}, g_wait_tag_offset{0u};
 unsigned exchange_max_polls() { return g_max_polls.load(std::memory_order_relaxed); }
 unsigned exchange_wait_tag_offset() { return g_wait_tag_offset.load(std::memory_order_relaxed); }
 
+int kl_advance_exchange_tags(unsigned used);  // reverse_kl_split.hip
+
 int open_split_exchange(ExchangeLaunch& x, hipStream_t stream, int64_t n_rows, bool own_ring_only) {
   return x.open<kRingWords>(split_family, reinterpret_cast<const void*>(&split_rings),
                             reinterpret_cast<const void*>(&split_topk_rings), kTopkRingWords, stream,
@@ -224,4 +226,11 @@ extern "C" int relax_amd_set_exchange_wait(int max_polls, int wait_tag_offset) {
   relax_amd::g_max_polls.store(max_polls == 0 ? relax_amd::kWaitPolls : unsigned(max_polls), std::memory_order_relaxed);
   relax_amd::g_wait_tag_offset.store(unsigned(wait_tag_offset), std::memory_order_relaxed);
   return RELAX_AMD_OK;
+}
+
+extern "C" int relax_amd_advance_exchange_tags(uint32_t used) {
+  using namespace relax_amd;
+  if (int rc = exchange_advance_tags<kRingWords>(split_family, reinterpret_cast<const void*>(&split_rings), used))
+    return rc;
+  return kl_advance_exchange_tags(used);
 }

@@ -257,6 +257,10 @@ namespace {
 ExchangeFamily kl_family{"reverse_kl_split", {}};
 }
 
+int kl_advance_exchange_tags(unsigned used) {
+  return exchange_advance_tags<kKlRingWords>(kl_family, reinterpret_cast<const void*>(&kl_split_rings), used);
+}
+
 // Long rows (12 and more vector positions per thread): three waves per SIMD, i.e. six workgroups per CU, each with
 // twelve teacher vectors per thread (24 KB) in LDS; with both rows in registers only two waves per SIMD fit, which is
 // 9 % slower on 16384 x 151936 rows (2.71 - 2.73 against 2.47 ms).  Shorter rows fit the registers of four and more

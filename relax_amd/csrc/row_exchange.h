@@ -135,6 +135,33 @@ struct ExchangeFamily {
   ExchangeDevice devices[kMaxDevices];
 };
 
+// relax_amd_advance_exchange_tags() for one family on the current device, which is idle: no ring goes back.
+template <size_t RING_WORDS>
+int exchange_advance_tags(ExchangeFamily& family, const void* ring_symbol, unsigned used) {
+  int index = -1;
+  void* rings = nullptr;
+  hipError_t e = hipGetDevice(&index);
+  if (e == hipSuccess && (index < 0 || index >= ExchangeFamily::kMaxDevices)) e = hipErrorInvalidDevice;
+  if (e == hipSuccess) e = hipGetSymbolAddress(&rings, ring_symbol);
+  unsigned counter = 0;
+  if (e == hipSuccess) {
+    unsigned* on_device = reinterpret_cast<unsigned*>(static_cast<unsigned long long*>(rings) +
+                                                      kCaptureRing * (RING_WORDS + kRingTailWords) + RING_WORDS);
+    e = hipMemcpy(&counter, on_device, sizeof(counter), hipMemcpyDeviceToHost);
+    if (e == hipSuccess && counter < used) e = hipMemcpy(on_device, &used, sizeof(used), hipMemcpyHostToDevice);
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    set_error("%s: exchange tags: %s", family.who, hipGetErrorString(e));
+    return RELAX_AMD_ELAUNCH;
+  }
+  for (RingTags& t : family.devices[index].tags) {
+    std::lock_guard<std::mutex> hold(t.lock);
+    if (t.used < used) t.used = used;
+  }
+  return RELAX_AMD_OK;
+}
+
 // The ring and the tags of one launch, held while it is enqueued.
 class ExchangeLaunch {
  public:

@@ -2109,6 +2109,55 @@ def test_one_shot_steps_of_two_threads_and_of_several_streams_stay_apart(v):
                 assert torch.equal(a, b), i
 
 
+def test_exchange_rings_are_cleared_before_a_tag_comes_round_again():
+    """The last tags of a ring and the first ones after its clearing, eager and in a graph's replays, three laps and one:
+    the two-walk kernels' bits.  Words of the rings' first launches, which carried the tags that come again, are other
+    inputs' sums, so that one taken for a neighbour's would show."""
+    from relax_amd import ops
+    from relax_amd._lib import check, lib
+
+    dev = require_gpu()
+    announce("exchange rings, tags at their end")
+    steps = [_any_row_step(v, torch.bfloat16, n, 0, 20 + i, dev)
+             for i, (v, n) in enumerate(((32000, 9000), (32000, 60), (16387, 300), (32000, 61)))]
+    wants = [step("two_walk")[1] for step in steps]
+    gen = torch.Generator(device=dev).manual_seed(9)
+    rows = [(torch.randn((50, 50304), device=dev, generator=gen) * 2).bfloat16() for _ in range(2)]
+    weight = torch.ones(50, device=dev)
+
+    def kl(kind="auto"):
+        ops.set_kernel_choice(kind)
+        out = ops.reverse_kl_step_fused(rows[0], rows[1], weight, 1.0)
+        ops.set_kernel_choice("auto")
+        return [out[0], out[3].view(torch.int16)]
+
+    want_kl = kl("two_walk")
+    for step in steps:
+        step()
+    kl(), kl()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        name, replayed = steps[1]()
+        replayed_kl = kl()
+    assert name == "actor_step_split"
+    graph.replay()
+    torch.cuda.synchronize()
+    check(lib.relax_amd_advance_exchange_tags(0xffffffff - 4))
+    for turn in range(4):
+        for i, (step, want) in enumerate(zip(steps, wants)):
+            for a, b in zip(want, step()[1]):
+                assert torch.equal(a, b), (turn, i)
+        graph.replay()
+        eager_kl = kl()
+        torch.cuda.synchronize()
+        for a, b in zip(wants[1], replayed):
+            assert torch.equal(a, b), (turn, "replay")
+        for got in (eager_kl, replayed_kl):
+            for a, b in zip(want_kl, got):
+                assert torch.equal(a, b), (turn, "reverse kl")
+
+
 @pytest.mark.parametrize("recorded", [1, 2])
 def test_captured_one_shot_steps_replayed_in_turn(recorded):
     """Graphs that record the same kernel family share a ring: each replay takes tags of its own."""
